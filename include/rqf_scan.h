@@ -357,8 +357,8 @@ int rqf_proj_gemm(const rqf_proj_gemm_args *args, rqf_stream_t stream);
  *   PAIRED    (Wr + i Wi) b for h the stacked real [Wr; Wi] (h_rows x w_cols),   *
  *             real b;                                                            *
  *   PAIRED_T  Re(W^H gz) for the same stack, gz complex (h_rows / 2 x n).        *
- * Matrices a mode does not use may be NULL.  The workspace (which may be 0       *
- * bytes) holds the weights split into bf16 parts.                                */
+ * Matrices a mode does not use may be NULL.  B has at least one row, or n or C     *
+ * none.  The workspace holds the weights split into bf16 parts.                  */
 #define RQF_PACK_FORWARD 0
 #define RQF_PACK_ADJOINT 1
 #define RQF_PACK_REAL 2

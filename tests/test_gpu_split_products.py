@@ -7,11 +7,13 @@ gives a 2-norm error below 2^-24 sqrt(K / 16 + 1) for products of random sign.  
 bar is four times that, against float64 on the same inputs.
 """
 
+import ctypes
 import math
 
 import pytest
 import torch
 
+from prospective_rqf_amd import _lib
 from prospective_rqf_amd import projection as P
 
 pytestmark = pytest.mark.gpu
@@ -210,3 +212,20 @@ def test_weight_gradient_of_complex_rows_against_real_ones():
     got = P.outer_sum(a, b)
     want = torch.cat((a.real, a.imag)).double() @ b.double().T
     assert _err(got, want) <= _bar(4100)
+
+
+@pytest.mark.parametrize("relu", [0, 1])
+@pytest.mark.parametrize("k_pad", [0, 16])
+def test_packed_product_over_nothing_is_the_bias(k_pad, relu):
+    weights = torch.ones(16, 128, device="cuda")
+    bias = torch.tensor([1.5, -2.0, 0.5], device="cuda")
+    z = torch.ones(2, 130, dtype=torch.complex64, device="cuda")
+    out = torch.ones(3, 130, device="cuda")
+    a = _lib.ProjGemmArgs()
+    a.weights, a.k_pad, a.m_pad, a.n = weights.data_ptr(), k_pad, 128, 130
+    a.out_cplx, a.out_cplx_rows = z.data_ptr(), 2
+    a.out_real, a.out_real_rows = out.data_ptr(), 3
+    a.out_real_bias, a.out_real_relu = bias.data_ptr(), relu
+    _lib.check(_lib.load().rqf_proj_gemm(ctypes.byref(a), _lib.stream_of(out)), "rqf_proj_gemm")
+    assert not z.any()
+    assert torch.equal(out, (bias.relu() if relu else bias)[:, None].expand(3, 130))
