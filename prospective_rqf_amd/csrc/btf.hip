@@ -173,7 +173,7 @@ __global__ __launch_bounds__(kThreads) void btf_fwd_kernel(
     if (PH == kChunks && l.fv) {
       const c64d ac = dpow(widen(a), sp.steps);
       for (int64_t j = 0; j < l.c; ++j)
-        cr = dmad(ac, cr, cd(tot[(l.b * sp.chunks + j) * F + l.f]));
+        cr = span_mad(ac, cr, cd(tot[(l.b * sp.chunks + j) * F + l.f]));
     }
     s_carry[0][l.fl] = d2(cr);
   }
@@ -295,7 +295,7 @@ __global__ __launch_bounds__(kThreads) void btf_bwd_kernel(
       chunk.c = mkd(pc.r * (double)sp.steps, pc.i * (double)sp.steps);
       for (int64_t j = sp.chunks - 1; j > l.c; --j) {
         const Pair t = tot[(l.b * sp.chunks + j) * F + l.f];
-        pair_apply(chunk, cd(t.g), cd(t.h), g, h);
+        pair_apply_span(chunk, cd(t.g), cd(t.h), g, h);
       }
     }
     s_carry[0][l.fl] = Pair{d2(g), d2(h)};

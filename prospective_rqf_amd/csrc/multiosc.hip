@@ -304,7 +304,7 @@ __global__ __launch_bounds__(W* kWave) void mosc_fwd_kernel(
       if (PH == kChunks && l.fv) {
         const c64d ac = dpow(widen(a[n]), sp.steps);
         for (int64_t j = 0; j < l.c; ++j)
-          cr = dmad(ac, cr, cd(tot[((l.b * sp.chunks + j) * F + l.f) * NP + n]));
+          cr = span_mad(ac, cr, cd(tot[((l.b * sp.chunks + j) * F + l.f) * NP + n]));
       }
       s_carry[0][n][l.fl] = d2(cr);
       s_k[n][l.fl] = fwd_maps<LS, W>(a[n]);
@@ -515,7 +515,7 @@ __global__ __launch_bounds__(kThreads) void mosc_bwd_kernel(
         chunk.c = mkd(pc.r * (double)sp.steps, pc.i * (double)sp.steps);
         for (int64_t j = sp.chunks - 1; j > l.c; --j) {
           const Pair t = tot[((l.b * sp.chunks + j) * F + l.f) * NP + n];
-          pair_apply(chunk, cd(t.g), cd(t.h), g, h);
+          pair_apply_span(chunk, cd(t.g), cd(t.h), g, h);
         }
       }
       s_carry[n][l.fl] = Pair{d2(g), d2(h)};

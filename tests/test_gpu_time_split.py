@@ -18,7 +18,11 @@ from prospective_rqf_amd.chunked_scan_kernel import (
     _triton_chunked_scan,
     _triton_chunked_scan_prospective,
 )
-from prospective_rqf_amd.multi_osc_scan import _forward
+from prospective_rqf_amd.multi_osc_scan import (
+    _forward,
+    _triton_sequential_scan_multi_osc,
+    _triton_sequential_scan_multi_osc_real,
+)
 from prospective_rqf_amd.scan import sequential_scan_abs
 from tests.helpers import PARITY_RTOL, chanerr, crandn, relerr
 from tests.test_gpu_multi_osc import (
@@ -103,3 +107,71 @@ def test_abs_readout(real):
 @pytest.mark.parametrize("N", [1, 2, 4])
 def test_multi_osc_gradient_subsets(N, real):
     _subsets_case((1, 2600, 18), N, real)
+
+
+# 64 sequences in chunks of eight passes (4096 steps): 1.25^4096 is past float64
+UNSTABLE = (64, 16000, 16)
+
+
+def _unstable(F):
+    return (1.25 * np.exp(0.3j * np.arange(F))).astype(np.complex64).astype(np.complex128)
+
+
+@pytest.mark.parametrize("prospective", [True, False])
+def test_unstable_filters_stay_finite_while_their_state_is_zero(prospective):
+    """Silence, then 50 steps: what whole sequences gave, from those steps alone."""
+    rng = np.random.default_rng(5)
+    (B, T, F), n = UNSTABLE, 50
+    _, t0, t1 = _coeffs(rng, F)
+    c1, t1 = _unstable(F), t1 if prospective else None
+    u, gy = _c64(crandn(rng, B, n, F)), _c64(crandn(rng, B, n, F))
+    leaves = [_dev(c) for c in (c1, t0) + ((t1,) if prospective else ())]
+    scan = _triton_chunked_scan_prospective if prospective else _triton_chunked_scan
+    x = torch.zeros(B, T, F, dtype=torch.complex64, device="cuda")
+    x[:, T - n:] = torch.as_tensor(u.astype(np.complex64))
+    with torch.no_grad():
+        y = scan(*leaves, x)
+    assert not y[:, :T - n].any()
+    assert relerr(y[:, T - n:], oracle.twotap_fwd(c1, t0, t1, u)) <= PARITY_RTOL
+    # the adjoint runs the other way: a cotangent of the first steps only
+    x = x.flip(1).contiguous().requires_grad_(True)
+    g = torch.zeros(B, T, F, dtype=torch.complex64, device="cuda")
+    g[:, :n] = torch.as_tensor(gy.astype(np.complex64))
+    scan(*leaves, x).backward(g)
+    u = u[:, ::-1]
+    gu, *gc = oracle.twotap_bwd(c1, t0, t1, u, oracle.twotap_fwd(c1, t0, t1, u), gy)
+    assert not x.grad[:, n:].any()
+    assert relerr(x.grad[:, :n], gu) <= PARITY_RTOL
+    for got, want in zip(leaves, gc):
+        assert relerr(got.grad, want) <= PARITY_RTOL
+
+
+@pytest.mark.parametrize("real", [False, True])
+@pytest.mark.parametrize("N", [1, 2, 4])
+def test_unstable_oscillators_stay_finite_while_their_state_is_zero(N, real):
+    """Each layout's whole-sequence result from the same steps (50 of them run whole)."""
+    rng = np.random.default_rng(6)
+    (B, T, F), n = UNSTABLE, 50
+    scan = _triton_sequential_scan_multi_osc_real if real else _triton_sequential_scan_multi_osc
+    c1 = _unstable(F * N)
+    c2, cw = _c64(crandn(rng, F * N)), torch.randn(F * N, 2, device="cuda")
+    u = torch.randn(B, n, F, dtype=torch.float32 if real else torch.complex64, device="cuda")
+    g = torch.randn(B, n, F, dtype=torch.complex64, device="cuda")
+
+    def run(x, gy):
+        leaves = [_dev(c1), _dev(c2), x.requires_grad_(True), cw.clone().requires_grad_(True)]
+        y = scan(*leaves, N)
+        return y.detach(), torch.autograd.grad(y, leaves, gy)
+
+    def padded(v, front):
+        out = torch.zeros(B, T, F, dtype=v.dtype, device="cuda")
+        (out[:, T - n:] if front else out[:, :n]).copy_(v)
+        return out
+
+    y, want = run(u.clone(), g)
+    late, _ = run(padded(u, True), padded(g, False))
+    assert not late[:, :T - n].any() and relerr(late[:, T - n:], y) <= PARITY_RTOL
+    _, got = run(padded(u, False), padded(g, False))
+    assert not got[2][:, n:].any()
+    for a, b in zip((got[0], got[1], got[2][:, :n], got[3]), want):
+        assert relerr(a, b) <= PARITY_RTOL
