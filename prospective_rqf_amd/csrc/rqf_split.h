@@ -5,10 +5,10 @@
 // bits are three times 8).  With |m| <= 2^-8 |x| and |l| <= 2^-17 |x|, a product
 // x y needs hh + hm + mh + mm + hl + lh; the three left out are below
 // 2^-24 |x y| together, and of random sign.  bf16 has float's exponents, so the last
-// part of a value below 2^-110 would fall under its smallest value: data operands
-// are split scaled by 2^16, which covers every normal float.  What is left is a value
-// past 2^111, an infinity or a NaN: their differences are NaN, the caller's sums too,
-// and it then takes the fp32 instructions.
+// part of a value below 2^-110 would fall under its smallest value: both operands
+// are split scaled by 2^16, which covers every normal float, and the sums carry 2^32.
+// What is left is a value past 2^111, a sum past 2^95, an infinity or a NaN: the scaled
+// sum is infinite or NaN, and the caller then takes the fp32 instructions.
 #pragma once
 
 #include "rqf_device.h"
@@ -20,7 +20,8 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr float kFltMax = 3.402823466e38f;
-constexpr float kSplitScale = 65536.0f, kSplitUnscale = 1.0f / 65536.0f;
+constexpr float kSplitScale = 65536.0f;  // of each operand
+constexpr float kSplitUnscale = 1.0f / kSplitScale / kSplitScale;  // of a sum of products
 
 // Eight values as three bf16 operands of an MFMA with 8 k per lane.
 struct Split8 {
@@ -49,16 +50,12 @@ __device__ __forceinline__ void split_pair(const float (&x)[8], int p, Split8& s
   s.m[p] = m;
   s.l[p] = pk_bf16(a, b);
 }
-__device__ __forceinline__ void split8(const float (&x)[8], Split8& s) {
-#pragma unroll
-  for (int p = 0; p < 4; ++p) split_pair(x, p, s);
-}
-
 __device__ __forceinline__ void split8_scaled(const float (&x)[8], Split8& s) {
   float y[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) y[j] = kSplitScale * x[j];
-  split8(y, s);
+#pragma unroll
+  for (int p = 0; p < 4; ++p) split_pair(y, p, s);
 }
 
 __device__ __forceinline__ v4f mfma_bf16(u32x4 a, u32x4 b, v4f c) {

@@ -201,7 +201,7 @@ __global__ __launch_bounds__(kThreadsW, 2) void wgrad_kernel(const WgradArgs g) 
     for (int j = 0; j < T; ++j)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        acc[i][j][v] = (acc[i][j][v] + low[i][j][v]) * (kSplitUnscale * kSplitUnscale);
+        acc[i][j][v] = (acc[i][j][v] + low[i][j][v]) * kSplitUnscale;
         finite = finite && fabsf(acc[i][j][v]) <= kFltMax;
       }
   const bool redo = __ballot(!finite) != 0;

@@ -124,6 +124,20 @@ def test_values_that_are_not_sums_of_three_parts(cplx, monkeypatch):
     assert _err(got[rows], w.to(wide)[rows] @ x.to(wide)) <= _bar(48)
 
 
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("exponent", [-100, -112, -116, -120, -125])
+def test_small_weights_keep_every_bit(exponent, packed):
+    """Weights whose last bits lie below bf16's smallest values, at the usual bar."""
+    g = _gen(64, 50, 3000)
+    w = torch.randn(50, 64, 2, generator=g, device="cuda").clamp_(-2, 2)
+    w = torch.view_as_complex((w + w.sign()) * 2.0 ** exponent)  # all normal
+    x = _rand(g, 64, 3000, cplx=True)
+    z, _ = P.fused_forward(x, w, None, P.pack_forward(w, None) if packed else None)
+    up = 2.0 ** -exponent
+    assert _err(z.to(torch.complex128) * up, (w.to(torch.complex128) * up) @ x.to(torch.complex128)
+                ) <= _bar(128)
+
+
 def test_everything_else_stays_on_torch(monkeypatch):
     """Forms the kernels do not serve: dtypes, strides, lazy conjugates, graphs of graphs,
     autocast, empty sizes, vectors."""
