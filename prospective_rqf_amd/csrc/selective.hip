@@ -1928,9 +1928,8 @@ int64_t fwd_blocks(const rqf_selective_inputs* in) {
 constexpr int kFwdMaxThreads = std::max(kFwdRbWaves, kFwdRbWavesRaw) * kWave;
 
 void launch_fwd(const rqf_selective_inputs* in, const float* z, const float* skip, float* raw,
-                float* act, float* entries, int chunk, int nc, bool vec, hipStream_t s) {
+                float* act, float* entries, int chunk, int nc, int waves, bool vec, hipStream_t s) {
   const dim3 grid((unsigned)(in->F * in->B));
-  const int waves = fwd_waves(in, (raw != nullptr && act != nullptr) || skip != nullptr);
   with_option_set(options_of(in), [&](auto oc) {
     constexpr int O = decltype(oc)::value;
     auto launch = [&](auto wc) {
@@ -2044,11 +2043,12 @@ int selective_fwd(const rqf_selective_inputs* in, const float* z, int64_t chunk,
   int st = check_inputs(in);
   if (st) return st;
   if (!z || !entries || (!raw && !act)) return RQF_ERR_ARG;
-  if (!grid_fits(fwd_blocks(in), kFwdMaxThreads)) return RQF_ERR_ARG;
+  const int waves = fwd_waves(in, (raw != nullptr && act != nullptr) || skip != nullptr);
+  if (!grid_fits(fwd_blocks(in), std::max(kFwdMaxThreads, waves * kWave))) return RQF_ERR_ARG;
   if (!aligned8(z) || !aligned8(skip) || !aligned8(raw) || !aligned8(act) || !aligned8(entries))
     return RQF_ERR_ALIGN;
   const int nc = (int)((in->T + chunk - 1) / chunk);
-  launch_fwd(in, z, skip, raw, act, entries, chunk_int(chunk), nc,
+  launch_fwd(in, z, skip, raw, act, entries, chunk_int(chunk), nc, waves,
              vec_ok(in, {z, skip, raw, act}), (hipStream_t)stream);
   return launch_status();
 }

@@ -111,6 +111,12 @@ def test_selective(lib, monkeypatch):
     assert rc == ERR_ARG, rc
 
 
+def test_selective_rows_forced_to_sixteen_wavefronts(lib, monkeypatch):
+    monkeypatch.setenv("RQF_FWD_WAVES", "few")
+    s = _selective((2**32 - 1) // 1024 // 8 + 1, 8, 2, 1)  # 1024-thread blocks
+    assert lib.rqf_selective_fwd(ctypes.byref(s), P, 256, P, P, P, None) == ERR_ARG
+
+
 def test_layer0_grads(lib):
     n = ((2**32 - 1) // 256 + 1) * 256 * 4  # 256-thread blocks of 4 columns each
     assert lib.rqf_layer0_grads(P, P, P, P, None, 4, 1, n, None, 0, None) == ERR_ARG
