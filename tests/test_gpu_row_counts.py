@@ -95,3 +95,16 @@ def test_selective_block_sizes_of_every_option_set(monkeypatch, waves, T, name, 
     activate, write_raw = OUTPUTS[out]
     run_case(3, 2, T, case, activate=activate, write_raw=write_raw, chunk=256, G=3, seed=T,
              **opts)
+
+
+@pytest.mark.parametrize("out", list(OUTPUTS))
+@pytest.mark.parametrize("name", list(SETS))
+@pytest.mark.parametrize("waves", ["narrow", "wide", "few"])
+@pytest.mark.parametrize("T", [1, 161, 511])
+def test_selective_rows_below_one_tile(monkeypatch, T, waves, name, out):
+    """Unaligned rows without a whole 512-step tile have kernels of their own."""
+    print(f"case: selective short T={T} {waves} {name} {out}", flush=True)
+    monkeypatch.setenv("RQF_FWD_WAVES", waves)
+    case, opts = SETS[name]
+    activate, write_raw = OUTPUTS[out]
+    run_case(3, 2, T, case, activate=activate, write_raw=write_raw, chunk=64, G=3, seed=T, **opts)
