@@ -1909,9 +1909,10 @@ int grp_force_timeout() {
 // or a skip tensor add streams.  The act-only contract at config 3's shape,
 // rotated runs on one box: 1.314 -> 1.282 ms with the narrow blocks.
 // Where the rows leave CUs idle, a block's own wavefronts are all that hides its
-// super-tiles' latency: up to two rows per CU take the wide blocks (F = 48, B = 7, T =
-// 7754 act only 26 -> 23 us), up to one per CU of more than a wide super-tile
-// kFwdRbWavesFew (F = 256, B = 1, T = 16000: 35 -> 32 us; two rows per CU lose, 26 ->
+// super-tiles' latency: up to two rows per CU of more than a narrow super-tile (2048
+// steps) take the wide blocks (F = 48, B = 7, T = 7754 act only 26 -> 23 us; F = 64, B = 8
+// narrow / wide: T = 300 6.5 / 7.1, 2000 9.5 / 9.7, 2100 12.8 / 11.2), up to one per CU of
+// more than a wide one kFwdRbWavesFew (F = 256, B = 1, T = 16000: 35 -> 32 us; two rows per CU lose, 26 ->
 // 30 at F = 48, B = 7).  RQF_FWD_WAVES=narrow|wide|few forces one (tests and tuning).
 int fwd_waves(const rqf_selective_inputs* in, bool extra_streams) {
   if (const char* e = std::getenv("RQF_FWD_WAVES")) {
@@ -1921,7 +1922,8 @@ int fwd_waves(const rqf_selective_inputs* in, bool extra_streams) {
   }
   const int64_t rows = in->F * in->B;
   if (rows <= kCus && in->T > kFwdRbWaves * kWave * kFwdK) return kFwdRbWavesFew;
-  return extra_streams || rows <= 2 * kCus ? kFwdRbWaves : kFwdRbWavesRaw;
+  if (rows <= 2 * kCus && in->T > kFwdRbWavesRaw * kWave * kFwdK) return kFwdRbWaves;
+  return extra_streams ? kFwdRbWaves : kFwdRbWavesRaw;
 }
 
 // Bound on the forward's grid: one block per row, the batch rounded up to kXcds chunks.
