@@ -21,6 +21,7 @@
 #include "rqf_device.h"
 #include "rqf_scan.h"
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -48,10 +49,12 @@ constexpr int kTiK = RQF_TI_K;
 constexpr int kTiTile = kWave * kTiK;
 constexpr int kTiWaves = 4;
 // Rows up to which a block takes twice the wavefronts forward (one block per CU), and
-// up to which the backward runs row blocks whatever the alignment: one wavefront per
-// row leaves most SIMDs empty there.  Backward, T = 15999 (us, per row / row block): 48
-// rows 78 / 27, 512 83 / 42, 1024 112 / 99, 2048 173 / 170; T = 1000: 1024 rows 19 / 19,
-// 2048 19 / 26.
+// up to which the backward may run row blocks whatever the alignment: one wavefront per
+// row leaves most SIMDs empty there.  A row block costs its setup whatever its length, so
+// the rows have to be long, the longer the more rows there are.  Backward (us, per row / row
+// block): 48 and 256 rows, T = 161 8.2 / 9.8, 500 9.6 / 9.8, 600 10.7 / 9.9; 512 rows, T =
+// 500 9.8 / 11.2, 1000 12.3 / 11.9, 2001 18.7 / 13.6; 1024 rows, T = 500 10.2 / 16.4, 2001
+// 20.3 / 20.8, 4001 31.9 / 29.0; T = 15999: 48 rows 78 / 27, 1024 112 / 99, 2048 173 / 170.
 constexpr int64_t kFewRows = 256, kFewBwdRows = 1024;
 
 __device__ __forceinline__ c32 ldc(const float* p, int64_t i) { return mk(p[2 * i], p[2 * i + 1]); }
@@ -758,8 +761,9 @@ int fbt_bwd(const float* c1, const float* t0, const float* t1, Drive drv, const 
       !aligned8(gout) || !aligned8(gz))
     return RQF_ERR_ALIGN;
   const int64_t R = F * B;
-  // the row-block backward on 2 KB-aligned or few rows, the per-row one otherwise
-  const bool rowblock = T % kTiTile == 0 || R <= kFewBwdRows;
+  // the row-block backward on 2 KB-aligned or few long rows, the per-row one otherwise
+  const bool rowblock =
+      T % kTiTile == 0 || (R <= kFewBwdRows && T > 2 * std::max(R, kFewRows));
   if (R > 0 && T > 0 &&
       !(rowblock ? grid_fits(R, kRbWaves * kWave)
                  : grid_fits((R + kTiWaves - 1) / kTiWaves, kTiWaves * kWave)))

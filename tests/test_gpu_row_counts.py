@@ -1,8 +1,8 @@
 """GPU parity of the row kernels by how many rows there are and how long they are.
 
 The forwards pick a block's wavefronts by the tiles of a row and by the rows against
-the 256 CUs, the FBT backward its form by the rows (one wavefront per row above 1024),
-and the selective kernels place (item, batch element) pairs for any batch size.  Every
+the 256 CUs, the FBT backward its form by the rows and their length (row blocks for at
+most 1024 rows of more than twice as many steps), and the selective kernels place (item, batch element) pairs for any batch size.  Every
 choice is checked against the fp64 oracle, at the bars of the other parity tests.
 """
 
@@ -33,7 +33,8 @@ def _need_gpu():
 # one to five 512-step tiles, two super-tiles of 16 wavefronts, and 1100 rows (the
 # backward with one wavefront per row; five rows per CU)
 SHAPES = [(3, 1, 161), (2, 2, 511), (2, 1, 513), (3, 1, 1025), (2, 1, 2049), (3, 1, 4097),
-          (2, 1, 8193), (550, 2, 301), (275, 4, 257)]
+          (2, 1, 8193), (550, 2, 301), (275, 4, 257), (300, 1, 599), (300, 1, 601),
+          (1023, 1, 2047)]
 
 
 @pytest.mark.parametrize("variant", ["raw", "act", "recompute", "layer0"])
