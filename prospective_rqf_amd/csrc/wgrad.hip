@@ -297,20 +297,24 @@ struct Plan {
   size_t bytes;
 };
 
-// Tiles of 128 x 128, or of 64 x 64 where those would be mostly padding (48 complex
-// channels: 96 x 96 real rows).
+// Tiles of 128 x 128, or of 64 x 64 where those would be mostly padding (192 x 128 real
+// rows) or, at the 128 columns a split of small tiles may have, too few blocks for the CUs:
+// real 264 x 256, n = 2048 23 us in 48 blocks of 128 x 128, 14 in 320 of 64 x 64; 520 x 512,
+// n = 2048 35 / 31; complex 48 x 48, n = 4000 22 / 10.
 Plan plan_of(int64_t mr, int64_t kr, int64_t n) {
   Plan p;
   const auto area = [&](int64_t r) { return (mr + r - 1) / r * ((kr + r - 1) / r) * r * r; };
-  p.t = 4 * area(64) <= 3 * area(128) ? 2 : 4;
+  const bool few = area(128) / (128 * 128) * (n / 128) < 512;
+  p.t = few || 4 * area(64) <= 3 * area(128) ? 2 : 4;
   const int64_t r = 32 * p.t;
   p.mt = (mr + r - 1) / r;
   p.kt = (kr + r - 1) / r;
-  // Three blocks for each of the 256 CUs, at most kSplitCols and at least 256
-  // columns each.
-  const int64_t fill = (768 + p.mt * p.kt - 1) / (p.mt * p.kt);
+  // Three blocks for each of the 256 CUs, at most kSplitCols columns each and at least 256,
+  // or 128 where that makes too few (real 16 x 16, n = 2048: 10.9 us with 256, 7.8 with 128).
+  const int64_t tiles = p.mt * p.kt, fill = (768 + tiles - 1) / tiles;
+  const int64_t least = p.t == 2 && tiles * (n / 128) < 512 ? 128 : 256;
   int64_t s = std::max(fill, (n + kSplitCols - 1) / kSplitCols);
-  s = std::max<int64_t>(1, std::min(s, n / 256));
+  s = std::max<int64_t>(1, std::min(s, n / least));
   p.cols = ((n + s - 1) / s + kStage - 1) / kStage * kStage;
   p.splits = p.cols ? (n + p.cols - 1) / p.cols : 0;
   p.bytes = sizeof(float) * (size_t)(p.splits * p.mt * r) * (size_t)(p.kt * r);

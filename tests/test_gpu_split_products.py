@@ -163,9 +163,11 @@ def test_everything_else_stays_on_torch(monkeypatch):
 
 
 # rows, rows, columns: a single product, below and past the 64- and 128-row tiles, a
-# last stage of 1 to 31 columns, several splits with a ragged last one.
+# last stage of 1 to 31 columns, several splits with a ragged last one, both tile sizes on
+# either side of 512 blocks.
 SUMS = [(1, 1, 1), (3, 33, 31), (16, 16, 2049), (31, 40, 4097), (65, 64, 5003), (48, 48, 60001),
-        (130, 20, 10304), (200, 129, 9000)]
+        (130, 20, 10304), (200, 129, 9000), (16, 16, 65535), (16, 16, 65536), (256, 256, 16383),
+        (256, 256, 16384)]
 
 
 @pytest.mark.parametrize("m,k,n", SUMS)
