@@ -245,3 +245,21 @@ def test_packed_product_over_nothing_is_the_bias(k_pad, relu):
     _lib.check(_lib.load().rqf_proj_gemm(ctypes.byref(a), _lib.stream_of(out)), "rqf_proj_gemm")
     assert not z.any()
     assert torch.equal(out, (bias.relu() if relu else bias)[:, None].expand(3, 130))
+
+
+# both sides of the narrow operand's limits, no column and one
+@pytest.mark.parametrize("f,d,n", [(64, 3, 1 << 18), (64, 3, (1 << 18) - 1), (64, 7, 1 << 18),
+                                   (64, 8, 1 << 18), (5, 3, 1), (5, 4, 300), (5, 3, 0)])
+def test_narrow_layer0_weight_gradient_copies_no_gradient(f, d, n):
+    g = _gen(f, d, n)
+    gz, h = _rand(g, f, n, cplx=True), _rand(g, d, n)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    got = P.real_weight_grad(gz, h)
+    used = torch.cuda.max_memory_allocated() - before
+    if n > 1000:
+        assert used < gz.numel() * 8
+    want = torch.cat((gz.real, gz.imag)).double() @ h.double().T
+    assert got.shape == (2 * f, d) and got.dtype is torch.float32
+    assert _err(got, want) <= _bar(2 * min(n, 4096)) if n else not got.any()
