@@ -380,7 +380,9 @@ int rqf_projection(int32_t mode, const float *w, int64_t w_rows, int64_t w_cols,
  *   real, complex     a [Re b; Im b]^T, fp32 (a_rows, 2 b_rows)                   *
  *   complex, real     [Re a; Im a] b^T, fp32 (2 a_rows, b_rows)                   *
  * Partial sums go through the workspace and are added in a fixed order, in fp64:  *
- * deterministic.  Sizes are positive.                                             */
+ * deterministic.  Sizes are positive.  The workspace (16-byte aligned) does not   *
+ * grow with n beyond 256 MB, or the real rows' products in fp32 if those are more, *
+ * and 16 bytes per element of out.                                                */
 size_t rqf_weight_grad_workspace(int64_t a_rows, int32_t a_cplx, int64_t b_rows, int32_t b_cplx,
                                  int64_t n);
 int rqf_weight_grad(const float *a, int64_t a_rows, int32_t a_cplx, const float *b, int64_t b_rows,

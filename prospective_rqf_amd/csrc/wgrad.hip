@@ -12,7 +12,9 @@
 //   complex . real:    [Re G; Im G] X^T  (rqf_models/ops/fbt_scan_kernel.py:993-996).
 //
 // The result is small and the sum is long, so the columns are cut into splits, one
-// block per (tile of P, split); the partial tiles are added in order, in fp64.
+// block per (tile of P, split); the partial tiles are added in order, in fp64.  Where all
+// of them would take much memory, the columns go through in passes of as many splits as
+// fit, each pass adding its tiles to fp64 sums.
 #include "rqf_device.h"
 #include "rqf_scan.h"
 #include "rqf_split.h"
@@ -42,10 +44,11 @@ struct WgradArgs {
   const float* b;
   int64_t ar, br;  // source rows
   int64_t n;
+  int64_t n0, n1;  // columns of this pass
   int64_t cols;    // columns per split, a multiple of kStage
   int64_t mt, kt;  // tiles of P
-  int64_t tiles;   // mt * kt * splits
-  float* partial;  // (splits, mt * 32 T, kt * 32 T)
+  int64_t tiles;   // mt * kt * splits of the pass
+  float* partial;  // (splits of the pass, mt * 32 T, kt * 32 T)
 };
 
 // Real row `row` of an operand at column n (fallback and tail).
@@ -74,7 +77,7 @@ __global__ __launch_bounds__(kThreadsW, 2) void wgrad_kernel(const WgradArgs g) 
   const int64_t id = xcd_contiguous(blockIdx.x, g.tiles);
   const int64_t per = g.mt * g.kt, split = id / per;
   const int64_t m0 = (id % per) / g.kt * kRows, k0 = (id % per) % g.kt * kRows;
-  const int64_t c0 = split * g.cols, c1 = std::min(c0 + g.cols, g.n);
+  const int64_t c0 = g.n0 + split * g.cols, c1 = std::min(c0 + g.cols, g.n1);
 
   // Thread t's pair u: group u % 4 of complex row u / 4, or of real rows u / 4 and
   // u / 4 + kRows / 2.  Rows past the end repeat the last one; they only reach
@@ -241,10 +244,12 @@ __global__ __launch_bounds__(kThreadsW, 2) void wgrad_kernel(const WgradArgs g) 
 // A block takes 16 elements of the output (a complex value counts as one); 16
 // threads share an element's splits, thread q adding q, q + 16, ... in order, so
 // that hundreds of splits of a small matrix do not make one long chain of loads.
+// sums: of several passes, the elements' sums of the passes before (after the first).
 template <bool AC, bool BC>
 __global__ __launch_bounds__(256) void wgrad_close_kernel(const float* __restrict__ partial,
                                                           int64_t splits, int64_t mp, int64_t ldp,
-                                                          int64_t ar, int64_t br,
+                                                          int64_t ar, int64_t br, bool first,
+                                                          bool last, double2* __restrict__ sums,
                                                           float* __restrict__ out) {
   __shared__ double s_sum[16][16][2];
   const int64_t rows = AC && !BC ? 2 * ar : ar, cols = BC && !AC ? 2 * br : br;
@@ -275,12 +280,15 @@ __global__ __launch_bounds__(256) void wgrad_close_kernel(const float* __restric
     s_sum[q][e][1] = im;
     __syncthreads();
     if (q == 0 && id < total) {
-      re = im = 0.0;
+      re = first ? 0.0 : sums[id].x;
+      im = first ? 0.0 : sums[id].y;
       for (int v = 0; v < 16; ++v) {
         re += s_sum[v][e][0];
         im += s_sum[v][e][1];
       }
-      if (AC && BC) {
+      if (!last) {
+        sums[id] = make_double2(re, im);
+      } else if (AC && BC) {
         out[2 * id] = (float)re;
         out[2 * id + 1] = (float)im;
       } else {
@@ -294,15 +302,22 @@ __global__ __launch_bounds__(256) void wgrad_close_kernel(const float* __restric
 struct Plan {
   int t;
   int64_t mt, kt, splits, cols;
+  int64_t per;   // splits per pass
+  size_t sums;   // bytes of the fp64 sums, before the partials; none for a single pass
   size_t bytes;
 };
+// The partial tiles of one pass, unless a split's alone are more: 4096 tiles of 128 x 128.
+// Complex 256 x 256 with n = 1024000 would take 512 MB at once, 4096 x 4096 134 GB.
+constexpr size_t kPassBytes = (size_t)256 << 20;
 
 // Tiles of 128 x 128, or of 64 x 64 where those would be mostly padding (192 x 128 real
 // rows) or, at the 128 columns a split of small tiles may have, too few blocks for the CUs:
 // real 264 x 256, n = 2048 23 us in 48 blocks of 128 x 128, 14 in 320 of 64 x 64; 520 x 512,
 // n = 2048 35 / 31; complex 48 x 48, n = 4000 22 / 10.
-Plan plan_of(int64_t mr, int64_t kr, int64_t n) {
+Plan plan_of(int64_t ar, bool ac, int64_t br, bool bc, int64_t n) {
   Plan p;
+  const int64_t mr = ac ? 2 * ar : ar, kr = bc ? 2 * br : br;
+  const int64_t outputs = ac && bc ? ar * br : mr * kr;
   const auto area = [&](int64_t r) { return (mr + r - 1) / r * ((kr + r - 1) / r) * r * r; };
   const bool few = area(128) / (128 * 128) * (n / 128) < 512;
   p.t = few || 4 * area(64) <= 3 * area(128) ? 2 : 4;
@@ -317,24 +332,35 @@ Plan plan_of(int64_t mr, int64_t kr, int64_t n) {
   s = std::max<int64_t>(1, std::min(s, n / least));
   p.cols = ((n + s - 1) / s + kStage - 1) / kStage * kStage;
   p.splits = p.cols ? (n + p.cols - 1) / p.cols : 0;
-  p.bytes = sizeof(float) * (size_t)(p.splits * p.mt * r) * (size_t)(p.kt * r);
+  const size_t split = sizeof(float) * (size_t)(p.mt * r) * (size_t)(p.kt * r);
+  const int64_t most = std::max<int64_t>(1, (int64_t)(kPassBytes / split));
+  const int64_t passes = std::max<int64_t>(1, (p.splits + most - 1) / most);
+  p.per = (p.splits + passes - 1) / passes;
+  p.sums = passes > 1 ? sizeof(double2) * (size_t)outputs : 0;
+  p.bytes = p.sums + split * (size_t)p.per;
   return p;
 }
 
 template <int T, bool AC, bool BC>
-int launch(const WgradArgs& g, const Plan& p, float* out, hipStream_t s) {
-  hipLaunchKernelGGL((wgrad_kernel<T, AC, BC>), dim3((unsigned)g.tiles), dim3(kThreadsW), 0, s, g);
+int launch(WgradArgs g, const Plan& p, double2* sums, float* out, hipStream_t s) {
   const int64_t total = (AC && !BC ? 2 : 1) * (BC && !AC ? 2 : 1) * g.ar * g.br;
-  hipLaunchKernelGGL((wgrad_close_kernel<AC, BC>), dim3(stride_blocks((total + 15) / 16)),
-                     dim3(256), 0, s, g.partial, p.splits, p.mt * 32 * T, p.kt * 32 * T, g.ar,
-                     g.br, out);
+  for (int64_t first = 0; first < p.splits; first += p.per) {
+    const int64_t splits = std::min(p.per, p.splits - first);
+    g.n0 = first * p.cols;
+    g.n1 = std::min(g.n0 + splits * p.cols, g.n);
+    g.tiles = p.mt * p.kt * splits;
+    hipLaunchKernelGGL((wgrad_kernel<T, AC, BC>), dim3((unsigned)g.tiles), dim3(kThreadsW), 0, s, g);
+    hipLaunchKernelGGL((wgrad_close_kernel<AC, BC>), dim3(stride_blocks((total + 15) / 16)),
+                       dim3(256), 0, s, g.partial, splits, p.mt * 32 * T, p.kt * 32 * T, g.ar, g.br,
+                       first == 0, first + p.per >= p.splits, sums, out);
+  }
   const hipError_t err = hipGetLastError();
   return err == hipSuccess ? RQF_OK : (int)err;
 }
 
 template <bool AC, bool BC>
-int launch(const WgradArgs& g, const Plan& p, float* out, hipStream_t s) {
-  return p.t == 4 ? launch<4, AC, BC>(g, p, out, s) : launch<2, AC, BC>(g, p, out, s);
+int launch(const WgradArgs& g, const Plan& p, double2* sums, float* out, hipStream_t s) {
+  return p.t == 4 ? launch<4, AC, BC>(g, p, sums, out, s) : launch<2, AC, BC>(g, p, sums, out, s);
 }
 
 }  // namespace
@@ -342,7 +368,7 @@ int launch(const WgradArgs& g, const Plan& p, float* out, hipStream_t s) {
 extern "C" size_t rqf_weight_grad_workspace(int64_t a_rows, int32_t a_cplx, int64_t b_rows,
                                             int32_t b_cplx, int64_t n) {
   if (a_rows < 1 || b_rows < 1 || n < 1) return 0;
-  return plan_of(a_cplx ? 2 * a_rows : a_rows, b_cplx ? 2 * b_rows : b_rows, n).bytes;
+  return plan_of(a_rows, a_cplx != 0, b_rows, b_cplx != 0, n).bytes;
 }
 
 extern "C" int rqf_weight_grad(const float* a, int64_t a_rows, int32_t a_cplx, const float* b,
@@ -351,9 +377,10 @@ extern "C" int rqf_weight_grad(const float* a, int64_t a_rows, int32_t a_cplx, c
   if (a_rows < 1 || b_rows < 1 || n < 1) return RQF_ERR_ARG;
   if (!a || !b || !out) return RQF_ERR_ARG;
   if (((uintptr_t)a | (uintptr_t)b | (uintptr_t)out) & 3) return RQF_ERR_ALIGN;
-  const Plan p = plan_of(a_cplx ? 2 * a_rows : a_rows, b_cplx ? 2 * b_rows : b_rows, n);
-  if (!grid_fits(p.mt * p.kt * p.splits, kThreadsW)) return RQF_ERR_ARG;
+  const Plan p = plan_of(a_rows, a_cplx != 0, b_rows, b_cplx != 0, n);
+  if (!grid_fits(p.mt * p.kt * p.per, kThreadsW)) return RQF_ERR_ARG;
   if (!workspace || workspace_bytes < p.bytes) return RQF_ERR_WORKSPACE;
+  if (p.sums && ((uintptr_t)workspace & 15)) return RQF_ERR_ALIGN;
   WgradArgs g;
   g.a = a;
   g.b = b;
@@ -363,10 +390,10 @@ extern "C" int rqf_weight_grad(const float* a, int64_t a_rows, int32_t a_cplx, c
   g.cols = p.cols;
   g.mt = p.mt;
   g.kt = p.kt;
-  g.tiles = p.mt * p.kt * p.splits;
-  g.partial = (float*)workspace;
+  double2* sums = (double2*)workspace;
+  g.partial = (float*)((char*)workspace + p.sums);
   hipStream_t s = (hipStream_t)stream;
   if (a_cplx)
-    return b_cplx ? launch<true, true>(g, p, out, s) : launch<true, false>(g, p, out, s);
-  return b_cplx ? launch<false, true>(g, p, out, s) : launch<false, false>(g, p, out, s);
+    return b_cplx ? launch<true, true>(g, p, sums, out, s) : launch<true, false>(g, p, sums, out, s);
+  return b_cplx ? launch<false, true>(g, p, sums, out, s) : launch<false, false>(g, p, sums, out, s);
 }

@@ -263,3 +263,25 @@ def test_narrow_layer0_weight_gradient_copies_no_gradient(f, d, n):
     want = torch.cat((gz.real, gz.imag)).double() @ h.double().T
     assert got.shape == (2 * f, d) and got.dtype is torch.float32
     assert _err(got, want) <= _bar(2 * min(n, 4096)) if n else not got.any()
+
+
+@pytest.mark.parametrize("ac,bc,m,k", [(False, False, 1100, 1030), (True, False, 550, 1030),
+                                       (False, True, 1100, 515), (True, True, 550, 515)])
+def test_weight_gradients_in_several_passes(ac, bc, m, k):
+    """74 splits of 5.3 MB run in two passes; an infinity in the second stays its own."""
+    n = 150001
+    print(f"case: weight gradient in passes {m} {k} {n} {ac} {bc}", flush=True)
+    g = _gen(m, k, ac, bc)
+    a, b = _rand(g, m, n, cplx=ac), _rand(g, k, n, cplx=bc)
+    got = P.outer_sum(a, b)
+    if ac and bc:
+        want = a.to(torch.complex128) @ b.to(torch.complex128).mH
+    else:
+        want = torch.cat((a.real, a.imag)).double() if ac else a.double()
+        want = want @ (torch.cat((b.real, b.imag)) if bc else b).double().T
+    assert _err(got, want) <= _bar(2 * 2048)
+    assert torch.equal(got, P.outer_sum(a, b))
+    (torch.view_as_real(a)[3, n - 2, 0] if ac else a[3, n - 2]).fill_(math.inf)
+    got = P.outer_sum(a, b)
+    rows = torch.arange(got.shape[0], device="cuda") != 3
+    assert not got[3].isfinite().any() and _err(got[rows], want[rows]) <= _bar(2 * 2048)
