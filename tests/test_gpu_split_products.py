@@ -222,6 +222,14 @@ def test_columns_past_a_descriptor():
     assert torch.equal(y, 3 * x)
 
 
+def test_packed_columns_past_a_descriptor():
+    n = P.MAX_COLS + 2
+    x = torch.ones(1, n, device="cuda")
+    x[0, 3], x[0, n - 1] = 2.5, -7.0
+    packed = P._padded(torch.tensor([[3.0]], device="cuda"))
+    assert torch.equal(P._proj_gemm(packed, None, x, n, 0, 1, x.device)[1], 3 * x)
+
+
 def test_weight_gradient_of_complex_rows_against_real_ones():
     g = _gen(11)
     a, b = _rand(g, 64, 4100, cplx=True), _rand(g, 128, 4100)
