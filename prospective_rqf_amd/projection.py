@@ -141,9 +141,12 @@ FORWARD, ADJOINT, REAL, REAL_T, PAIRED, PAIRED_T = range(6)
 # the multiplications, weight size times columns, from which two launches of these
 # kernels beat the library's one: complex 48 x 48 weights, 5000 columns 13.0 against
 # 11.7 us, 10304 13.1 against 15.8; real 520 x 512, 2500 columns 28 against 23 us,
-# 10304 47 against 78.
+# 10304 47 against 78.  A block walks the inner dimension in series (40 us at 1024), so from
+# 512 on real products need as many times more of them: 1032 x 1024, 1288 columns 45
+# against 32 us, 2576 56 against 53, 5152 72 against 108.
 MAX_SIDE, MAX_COLS = 8192, (1 << 25) - 1
 MIN_WORK = {torch.complex64: 1 << 24, torch.float32: 1 << 30}
+REAL_INNER = 512
 _PLAIN = (Tensor, torch.nn.Parameter)
 
 
@@ -153,8 +156,11 @@ def _kernel_serves(weight: Tensor, x: Tensor) -> bool:
     contiguous, and nothing recorded, traced, batched (those tensors have no storage of
     their own) or autocast.  Everything else stays on torch."""
     dt = x.dtype
-    if (dt not in MIN_WORK or x.dim() != 2 or weight.dim() != 2
-            or weight.numel() * x.shape[1] < MIN_WORK[dt]):
+    if dt not in MIN_WORK or x.dim() != 2 or weight.dim() != 2:
+        return False
+    work = weight.numel() * x.shape[1]
+    if work < MIN_WORK[dt] or (dt is torch.float32
+                               and work * REAL_INNER < MIN_WORK[dt] * x.shape[0]):
         return False
     return (
         weight.dtype is dt and weight.numel() > 0 and 0 < x.shape[1] <= MAX_COLS

@@ -138,6 +138,21 @@ def test_small_weights_keep_every_bit(exponent, packed):
                 ) <= _bar(128)
 
 
+@pytest.mark.parametrize("m,k,n,kernel", [(1024, 1024, 1024, False), (1024, 1024, 2047, False),
+                                          (1024, 1024, 2048, True), (512, 512, 4095, False),
+                                          (512, 512, 4096, True), (256, 256, 16384, True)])
+def test_long_inner_dimensions_need_more_columns(m, k, n, kernel, monkeypatch):
+    taken = []
+    gemm = P.gemm
+    monkeypatch.setattr(P, "gemm", lambda *a, **kw: taken.append(a[0]) or gemm(*a, **kw))
+    g = _gen(m, k, n)
+    w, x, y = _rand(g, m, k), _rand(g, k, n), _rand(g, m, n)
+    got = P.matmul(w, x), P.matmul_adjoint(w, y)
+    assert taken == ([P.REAL, P.REAL_T] if kernel else [])
+    for a, want in zip(got, (w.double() @ x.double(), w.double().T @ y.double())):
+        assert _err(a, want) <= 4 * 2.0 ** -24 * math.sqrt(k)
+
+
 def test_everything_else_stays_on_torch(monkeypatch):
     """Forms the kernels do not serve: dtypes, strides, lazy conjugates, graphs of graphs,
     autocast, empty sizes, vectors."""
