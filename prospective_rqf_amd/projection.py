@@ -27,6 +27,7 @@ import ctypes
 
 import torch
 from torch import Tensor
+from torch.autograd import forward_ad
 
 # Batched GEMMs the reduction is split into, and the least columns per split.
 # Measured on MI355X for (out, in, batch*time) = (256, 256, 1.02e6):
@@ -55,6 +56,7 @@ def _wgrad_serves(g: Tensor, x: Tensor, columns: int = WGRAD_KERNEL_COLUMNS,
                 for t in (g, x))
         and not (torch.is_grad_enabled() and (g.requires_grad or x.requires_grad))
         and not torch.is_autocast_enabled("cuda")
+        and forward_ad._current_level < 0
         and not torch.compiler.is_compiling()
     )
 
@@ -154,7 +156,8 @@ def _kernel_serves(weight: Tensor, x: Tensor) -> bool:
     """Whether a product of these runs on the kernels: plain float32 or complex64
     matrices of one dtype on the current device, enough work, the data ``x``
     contiguous, and nothing recorded, traced, batched (those tensors have no storage of
-    their own) or autocast.  Everything else stays on torch."""
+    their own) or autocast, nor a level of dual numbers open, whose tangents the kernels
+    would drop.  Everything else stays on torch."""
     dt = x.dtype
     if dt not in MIN_WORK or x.dim() != 2 or weight.dim() != 2:
         return False
@@ -172,6 +175,7 @@ def _kernel_serves(weight: Tensor, x: Tensor) -> bool:
         and x.is_contiguous() and not x.is_conj() and not x.is_neg()
         and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
         and not torch.is_autocast_enabled("cuda")
+        and forward_ad._current_level < 0
         and not torch.compiler.is_compiling()
     )
 

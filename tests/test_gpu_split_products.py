@@ -12,6 +12,7 @@ import math
 
 import pytest
 import torch
+from torch.autograd import forward_ad
 
 from prospective_rqf_amd import _lib
 from prospective_rqf_amd import projection as P
@@ -308,3 +309,21 @@ def test_weight_gradients_in_several_passes(ac, bc, m, k):
     got = P.outer_sum(a, b)
     rows = torch.arange(got.shape[0], device="cuda") != 3
     assert not got[3].isfinite().any() and _err(got[rows], want[rows]) <= _bar(2 * 2048)
+
+
+def test_forward_mode_keeps_its_tangents():
+    """Dual cotangents through a backward (forward over reverse), and the products
+    themselves: at these sizes the kernels serve otherwise."""
+    g = _gen(15)
+    v, w = _rand(g, 512, 8192).requires_grad_(), _rand(g, 520, 512).requires_grad_()
+    (y,) = P.split_projection(v, w, (520,))
+    gy, ty = _rand(g, 520, 8192), _rand(g, 520, 8192)
+    with forward_ad.dual_level():
+        dual = forward_ad.make_dual(gy, ty)
+        got = [forward_ad.unpack_dual(t).tangent for t in (
+            *torch.autograd.grad(y, (v, w), dual), P.weight_grad(dual, v.detach()),
+            P.matmul_adjoint(w.detach(), dual))]
+    dv, dw = w.detach().double().T @ ty.double(), ty.double() @ v.detach().double().T
+    for t, want in zip(got, (dv, dw, dw, dv)):
+        # the library may add one product at a time: N additions, not N / 16
+        assert t is not None and _err(t, want) <= _bar(16 * 8192)
