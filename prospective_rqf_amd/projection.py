@@ -312,8 +312,8 @@ def gemm(mode: int, weight: Tensor | None, heads: Tensor | None, b_cplx: Tensor 
     n, device = b.shape[1], b.device
     w, h = weight, heads
     if w is not None and not (w.dtype is torch.complex64 and w.is_contiguous()
-                              and not w.is_conj()):
-        w = w.to(torch.complex64).resolve_conj().contiguous()
+                              and not w.is_conj() and not w.is_neg()):
+        w = w.to(torch.complex64).resolve_conj().resolve_neg().contiguous()
     if h is not None and not (h.dtype is torch.float32 and h.is_contiguous()
                               and not h.is_neg()):
         h = h.float().resolve_neg().contiguous()

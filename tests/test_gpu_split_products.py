@@ -327,3 +327,15 @@ def test_forward_mode_keeps_its_tangents():
     for t, want in zip(got, (dv, dw, dw, dv)):
         # the library may add one product at a time: N additions, not N / 16
         assert t is not None and _err(t, want) <= _bar(16 * 8192)
+
+
+def test_lazily_negated_weights():
+    g = _gen(16)
+    w, x, h = _rand(g, 40, 24, cplx=True), _rand(g, 24, 20000, cplx=True), _rand(g, 7, 48)
+    want = -w.to(torch.complex128) @ x.to(torch.complex128)
+    neg = torch._neg_view(w)
+    assert neg.is_neg() and _err(P.matmul(neg, x), want) <= _bar(48)
+    z, logits = P.fused_forward(x, neg, torch._neg_view(h))
+    assert _err(z, want) <= _bar(48)
+    v = torch.cat((x.real, x.imag)).double()
+    assert _err(logits, -h.double() @ v) <= _bar(48)
