@@ -830,7 +830,8 @@ void launch_fwd(const float* c1, const float* c2, const float* cw, const float* 
   if constexpr (!G64) {
     if (sp.chunks > 1) {
       const dim3 few(kSplitWaves * kWave);
-      hipLaunchKernelGGL((mosc_fwd_kernel<NP, REAL, true, false, kSplitWaves, false, kTotals>),
+      // The end states need no output weights: the form without C-weights, for any N.
+      hipLaunchKernelGGL((mosc_fwd_kernel<NP, REAL, false, false, kSplitWaves, false, kTotals>),
                          dim3((unsigned)(blocks * (sp.chunks - 1))), few, 0, s, c1, c2, nullptr, u,
                          yin, yout, T, F, N, n0, sp, tot);
       const dim3 all((unsigned)(blocks * sp.chunks));
