@@ -24,31 +24,10 @@ from prospective_rqf_amd.projection import (
     ADJOINT,
     FORWARD,
     _PLAIN,
-    _padded,
     gemm,
     real_weight_grad,
     weight_grad,
 )
-
-
-def pack_hidden(w1: Tensor) -> Tensor:
-    """A of ``W1 [Re f; Im f]`` over the interleaved K order (re f_0, im f_0, ...)."""
-    h, f2 = w1.shape
-    f = f2 // 2
-    a = torch.empty(h, f2, dtype=torch.float32, device=w1.device)
-    a[:, 0::2], a[:, 1::2] = w1[:, :f].float(), w1[:, f:].float()
-    return _padded(a)
-
-
-def pack_feature_grad(w1: Tensor) -> Tensor:
-    """A of the feature gradient ``W1^T dh`` as complex rows: row 2f is its real
-    part ``sum_h W1[h, f] dh_h``, row 2f + 1 its imaginary part
-    ``sum_h W1[h, F + f] dh_h``."""
-    h, f2 = w1.shape
-    f = f2 // 2
-    a = torch.empty(f2, h, dtype=torch.float32, device=w1.device)
-    a[0::2], a[1::2] = w1[:, :f].T.float(), w1[:, f:].T.float()
-    return _padded(a)
 
 
 # Most classes that rqf_readout_grads takes.

@@ -153,7 +153,6 @@ def _kernel_emulation(packed, b_cplx, b_real, out_cplx_rows, out_real_rows):
 
 def test_packed_weights_give_the_reference_products():
     from prospective_rqf_amd.projection import pack_dx, pack_forward
-    from prospective_rqf_amd.readout import pack_feature_grad, pack_hidden
 
     gen = torch.Generator().manual_seed(11)
     F, D, ml, N = 5, 3, 7, 13
@@ -170,14 +169,15 @@ def test_packed_weights_give_the_reference_products():
     dv = Ws64.T @ g.double()
     want = W64.mH @ dz.to(torch.complex128) + torch.complex(dv[:D], dv[D:])
     assert torch.allclose(dx, want, atol=1e-9)
-    # Readout: hidden = W1 [Re f; Im f]; the feature gradient W1^T dh as complex rows.
+    # The readout's two products are these layouts without a complex weight: hidden =
+    # W1 [Re f; Im f], and the feature gradient W1^T dh as complex rows.
     H = 4
     w1 = torch.randn(H, 2 * F, generator=gen)
     f = _rand((F, N), True, gen)
-    _, hid = _kernel_emulation(pack_hidden(w1), f, None, 0, H)
+    _, hid = _kernel_emulation(pack_forward(_rand((0, F), True, gen), w1), f, None, 0, H)
     f64 = f.to(torch.complex128)
     assert torch.allclose(hid, w1.double() @ torch.cat((f64.real, f64.imag), 0), atol=1e-9)
     dh = torch.randn(H, N, generator=gen)
-    df, _ = _kernel_emulation(pack_feature_grad(w1), None, dh, F, 0)
+    df, _ = _kernel_emulation(pack_dx(_rand((0, F), True, gen), w1), None, dh, F, 0)
     dfv = w1.double().T @ dh.double()
     assert torch.allclose(df, torch.complex(dfv[:F], dfv[F:]), atol=1e-9)
