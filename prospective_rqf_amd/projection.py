@@ -37,6 +37,14 @@ WGRAD_SPLITS = 128
 WGRAD_MIN_COLUMNS = 1024
 
 
+def unobserved() -> bool:
+    """Whether plain tensors are all there is to a call: no open level of dual numbers,
+    whose tangents a kernel would drop, and no tracer or dispatch mode, which would take
+    its result for a constant."""
+    return (forward_ad._current_level < 0 and not torch._C._is_tracing()
+            and torch._C._len_torch_dispatch_stack() == 0 and not torch.compiler.is_compiling())
+
+
 # Columns and matrix side from which the kernel beats the batched GEMMs: complex 48 x 48,
 # 4000 columns 23 against 49 us; real 520 x 512, 1000 columns 35 against 21 us, 4000 42
 # against 56; real 10 x 256, 512000 columns 146 against 122 us.
@@ -56,8 +64,7 @@ def _wgrad_serves(g: Tensor, x: Tensor, columns: int = WGRAD_KERNEL_COLUMNS,
                 for t in (g, x))
         and not (torch.is_grad_enabled() and (g.requires_grad or x.requires_grad))
         and not torch.is_autocast_enabled("cuda")
-        and forward_ad._current_level < 0
-        and not torch.compiler.is_compiling()
+        and unobserved()
     )
 
 
@@ -155,9 +162,9 @@ _PLAIN = (Tensor, torch.nn.Parameter)
 def _kernel_serves(weight: Tensor, x: Tensor) -> bool:
     """Whether a product of these runs on the kernels: plain float32 or complex64
     matrices of one dtype on the current device, enough work, the data ``x``
-    contiguous, and nothing recorded, traced, batched (those tensors have no storage of
-    their own) or autocast, nor a level of dual numbers open, whose tangents the kernels
-    would drop.  Everything else stays on torch."""
+    contiguous, and nothing recorded, traced or in forward mode (``unobserved``), batched
+    (those tensors have no storage of their own) or autocast.  Everything else stays on
+    torch."""
     dt = x.dtype
     if dt not in MIN_WORK or x.dim() != 2 or weight.dim() != 2:
         return False
@@ -175,8 +182,7 @@ def _kernel_serves(weight: Tensor, x: Tensor) -> bool:
         and x.is_contiguous() and not x.is_conj() and not x.is_neg()
         and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
         and not torch.is_autocast_enabled("cuda")
-        and forward_ad._current_level < 0
-        and not torch.compiler.is_compiling()
+        and unobserved()
     )
 
 

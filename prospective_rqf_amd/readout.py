@@ -18,7 +18,6 @@ from __future__ import annotations
 
 import torch
 from torch import Tensor
-from torch.autograd import forward_ad
 
 from prospective_rqf_amd.projection import (
     ADJOINT,
@@ -26,6 +25,7 @@ from prospective_rqf_amd.projection import (
     _PLAIN,
     gemm,
     real_weight_grad,
+    unobserved,
     weight_grad,
 )
 
@@ -43,7 +43,7 @@ def _head_grads(dlogits: Tensor, hidden: Tensor, w2: Tensor):
     (c, n), rows = dlogits.shape, w2.shape[1]
     if not (0 < c <= _MAX_CLASSES and 0 < rows <= 1 << 20 and n > 0
             and hidden.shape == (rows, n) and hidden.dtype is torch.float32
-            and forward_ad._current_level < 0
+            and unobserved()
             and all(type(t) in _PLAIN and t.is_cuda and t.is_contiguous() and not t.is_neg()
                     and t.get_device() == torch._C._cuda_getDevice()
                     and torch._C._has_storage(t) for t in (dlogits, hidden, w2))):

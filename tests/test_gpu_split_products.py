@@ -13,6 +13,7 @@ import math
 import pytest
 import torch
 from torch.autograd import forward_ad
+from torch.fx.experimental.proxy_tensor import make_fx
 
 from prospective_rqf_amd import _lib
 from prospective_rqf_amd import projection as P
@@ -339,3 +340,26 @@ def test_lazily_negated_weights():
     assert _err(z, want) <= _bar(48)
     v = torch.cat((x.real, x.imag)).double()
     assert _err(logits, -h.double() @ v) <= _bar(48)
+
+
+@pytest.mark.parametrize("tracer", ["jit", "fx"])
+def test_traces_hold_the_products(tracer):
+    """A trace of products that the kernels serve, run on other data."""
+    g = _gen(17)
+    w, x, y = (_rand(g, *s, cplx=True) for s in ((64, 64), (64, 20000), (64, 20000)))
+
+    def products(w, x, y):
+        leaf = w.detach().requires_grad_()
+        out = [P.matmul(w, x), P.matmul_adjoint(w, x), P.weight_grad(x, y)]
+        if tracer == "fx":
+            out += torch.autograd.grad(P.project(leaf, x), leaf, y)
+        return out
+
+    trace = (make_fx(products)(w, x, y) if tracer == "fx"
+             else torch.jit.trace(products, (w, x, y), check_trace=False))
+    other = [_rand(g, *t.shape, cplx=True) for t in (w, x, y)]
+    w64, x64, y64 = (t.to(torch.complex128) for t in other)
+    wants = [w64 @ x64, w64.mH @ x64, x64 @ y64.mH, y64 @ x64.mH]
+    for got, want in zip(trace(*other), wants):
+        # the library may add one product at a time: N additions, not N / 16
+        assert _err(got, want) <= _bar(16 * 40000)
