@@ -1178,7 +1178,9 @@ __global__ __launch_bounds__(kTeam* kWave)
   __shared__ double s_sum[kChans][2];              // dbias, dtheta sums of finished segments
   const int lane = lane_id();
   const int w = wave_id();
-  const ItemId id = item_id(tm.slots, p.B, xcd_remap(blockIdx.x, gridDim.x));
+  const int64_t L = xcd_remap(blockIdx.x, gridDim.x);
+  if (L >= (int64_t)tm.slots * p.B) return;  // block-uniform: the other XCDs of bwd_one_xcd
+  const ItemId id = item_id(tm.slots, p.B, L);
   const int slot = (int)id.item;
   const int64_t b = id.b;
   if (slot >= *tm.nsplits) return;  // block-uniform
@@ -2180,6 +2182,19 @@ SelWs sel_ws_layout(const rqf_selective_inputs* in, int64_t chunk, bool group_fo
   return w;
 }
 
+// Whether the split form's blocks all run on one XCD: of one short recording, where
+// reading the team tables and the split partials back through one L2 is worth more than
+// the other CUs, the more so the more partials share a warp row.  The launch then has
+// kXcds times the blocks and the XCD-contiguous order leaves all but the first XCD's
+// idle.  One recording, spread / on one XCD (us): G = 1, F = 128, T = 161 23.4 / 19.1, F =
+// 256, T = 300 35.7 / 30.3, F = 256, T = 400 35.6 / 40.6, F = 64, T = 1000 27.1 / 24.3,
+// 1500 33.3 / 36.9; G = 2, F = 128, T = 400 21.7 / 18.6, F = 256, T = 161 24.5 / 26.0; G =
+// 4, F = 256, T = 100 19.3 / 17.4, 161 20.7 / 22.3; G = 8, F = 64, T = 400 17.3 / 16.9, F =
+// 200, T = 161 18.0 / 19.3.
+bool bwd_one_xcd(const rqf_selective_inputs* in) {
+  return in->B == 1 && in->F * in->T <= (in->has_warp && in->G <= 2 ? 80000 : 30000);
+}
+
 // Every grid a non-empty backward launches, within one dispatch's work-item
 // count: the tile-entry rebuild (chunk > one tile), the group form's (group,
 // batch element) blocks or the split form's team blocks, and the finishing
@@ -2326,7 +2341,8 @@ extern "C" int rqf_selective_bwd(const rqf_selective_inputs* in, const float* z,
     tm.gteam = gteam;
     tm.slots = w.split_slots;
     o.dd_part = in->has_warp ? (float*)(ws + w.dd) : nullptr;
-    const dim3 grid((unsigned)(w.split_slots * in->B)), block(kTeam * kWave);
+    const dim3 grid((unsigned)((bwd_one_xcd(in) ? kXcds : 1) * w.split_slots * in->B)),
+        block(kTeam * kWave);
     with_option_set(options_of(in), [&](auto oc) {
       constexpr int O = decltype(oc)::value;
       with_cotangent_set(cotangent_set(O, vec, gy, gx, truncated), [&](auto cc) {

@@ -109,3 +109,12 @@ def test_selective_rows_below_one_tile(monkeypatch, T, waves, name, out):
     case, opts = SETS[name]
     activate, write_raw = OUTPUTS[out]
     run_case(3, 2, T, case, activate=activate, write_raw=write_raw, chunk=64, G=3, seed=T, **opts)
+
+
+@pytest.mark.parametrize("F,T,G", [(16, 100, 1), (40, 2000, 1), (40, 2001, 1), (30, 1000, 3),
+                                   (30, 1001, 3)])
+def test_selective_one_recording(F, T, G):
+    """The backward of one short recording runs on one XCD, up to 80000 steps of all
+    channels with one or two warp rows, else 30000."""
+    print(f"case: selective one recording {F} {T} {G}", flush=True)
+    run_case(F, 1, T, CASE_ALL, G=G, seed=T)
