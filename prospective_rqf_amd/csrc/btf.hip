@@ -172,8 +172,11 @@ __global__ __launch_bounds__(kThreads) void btf_fwd_kernel(
     c64d cr = mkd(0.0, 0.0);
     if (PH == kChunks && l.fv) {
       const c64d ac = dpow(widen(a), sp.steps);
-      for (int64_t j = 0; j < l.c; ++j)
-        cr = span_mad(ac, cr, cd(tot[(l.b * sp.chunks + j) * F + l.f]));
+      int64_t first = 0;
+      if (!is_finite(ac))
+        while (first < l.c && is_zero(cr)) cr = cd(tot[(l.b * sp.chunks + first++) * F + l.f]);
+      for (int64_t j = first; j < l.c; ++j)
+        cr = dmad(ac, cr, cd(tot[(l.b * sp.chunks + j) * F + l.f]));
     }
     s_carry[0][l.fl] = d2(cr);
   }
@@ -293,9 +296,15 @@ __global__ __launch_bounds__(kThreads) void btf_bwd_kernel(
       PairMap chunk;
       chunk.P = dmul(pc, widen(ac));
       chunk.c = mkd(pc.r * (double)sp.steps, pc.i * (double)sp.steps);
-      for (int64_t j = sp.chunks - 1; j > l.c; --j) {
+      int64_t last = sp.chunks - 1;
+      if (!is_finite(chunk.P) || !is_finite(chunk.c))
+        for (; last > l.c && is_zero(g) && is_zero(h); --last) {
+          g = cd(tot[(l.b * sp.chunks + last) * F + l.f].g);
+          h = cd(tot[(l.b * sp.chunks + last) * F + l.f].h);
+        }
+      for (int64_t j = last; j > l.c; --j) {
         const Pair t = tot[(l.b * sp.chunks + j) * F + l.f];
-        pair_apply_span(chunk, cd(t.g), cd(t.h), g, h);
+        pair_apply(chunk, cd(t.g), cd(t.h), g, h);
       }
     }
     s_carry[0][l.fl] = Pair{d2(g), d2(h)};

@@ -94,10 +94,9 @@ __device__ __forceinline__ c64d dmul(c64d a, c64d b) {
 __device__ __forceinline__ c64d dmad(c64d a, c64d b, c64d c) {
   return mkd(fma(a.r, b.r, fma(-a.i, b.i, c.r)), fma(a.r, b.i, fma(a.i, b.r, c.i)));
 }
-// a b + c for the power a of a long span, which may overflow: a zero state b stays zero
-// through it.
-__device__ __forceinline__ c64d span_mad(c64d a, c64d b, c64d c) {
-  return b.r == 0.0 && b.i == 0.0 ? c : dmad(a, b, c);
+__device__ __forceinline__ bool is_zero(c64d a) { return a.r == 0.0 && a.i == 0.0; }
+__device__ __forceinline__ bool is_finite(c64d a) {
+  return fabs(a.r) <= 1.7976931348623157e308 && fabs(a.i) <= 1.7976931348623157e308;
 }
 // a^n, n >= 0, by binary powering in fp64.
 __device__ __forceinline__ c64d dpow(c64d a, int64_t n) {
@@ -551,14 +550,6 @@ __device__ __forceinline__ PairMap pair_map_mul(PairMap x, PairMap y) {
 __device__ __forceinline__ void pair_apply(const PairMap& mp, c64d G, c64d H, c64d& g, c64d& h) {
   const c64d ng = dmad(mp.P, g, G);
   h = dmad(mp.P, h, dmad(mp.c, g, H));
-  g = ng;
-}
-
-// The same across a span whose powers may overflow.
-__device__ __forceinline__ void pair_apply_span(const PairMap& mp, c64d G, c64d H, c64d& g,
-                                                c64d& h) {
-  const c64d ng = span_mad(mp.P, g, G);
-  h = span_mad(mp.P, h, span_mad(mp.c, g, H));
   g = ng;
 }
 

@@ -7,9 +7,9 @@
 // state only (its pair at its start, for an adjoint), the second forms each chunk's
 // entry from the chunks before (after) it, in fp64 with the power of the chunk's
 // length, and runs the chunk.  An unstable filter's power may overflow (|c1| = 1.2 at 4096
-// steps), so it never multiplies a zero: silence before a chunk stays silence, as it does
-// in a whole sequence.  The input is read twice, so large grids, which memory
-// bounds, run whole sequences.
+// steps), so there the entry starts from the first state that is not zero: silence before a
+// chunk stays silence, as it does in a whole sequence.  The input is read twice, so large
+// grids, which memory bounds, run whole sequences.
 #pragma once
 
 #include <stdint.h>
